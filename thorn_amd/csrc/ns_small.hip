@@ -679,30 +679,26 @@ __device__ __forceinline__ float small_momentum_tile(const OrthoMat& M, int t, i
     float nrm = 0.f;
 #pragma unroll
     for (int rr = 0; rr < 4; ++rr) {
+        [[maybe_unused]] const float before[4] = {mv[rr][0], mv[rr][1], mv[rr][2], mv[rr][3]};
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             mv[rr][e] = mv[rr][e] * beta1 + gv[rr][e];
             const float x = fmaf(mv[rr][e], beta1, gv[rr][e]);
             nrm += x * x;   // (zeros outside the matrix)
-            if constexpr (KEEP && BF) {   // as u_of makes it from what store_moment keeps
-                const unsigned short h = bf16_round(mv[rr][e]);
-                u[4 * rr + e] = fmaf(bf16_restore(h, bf16_residual(mv[rr][e], h)), beta1, gv[rr][e]);
-            } else if constexpr (KEEP) {
-                u[4 * rr + e] = x;
-            }
+            if constexpr (KEEP) u[4 * rr + e] = x;
         }
         if (vec) {
             const int row = tm.row(rr, 4 * lane), c = tm.col(4 * lane);
             if (row >= M.rows || c >= M.cols) continue;
             const float4 m = make_float4(mv[rr][0], mv[rr][1], mv[rr][2], mv[rr][3]);
-            if constexpr (BF && !KEEP) store_moment4(M, row, c, m);
+            if constexpr (BF && !KEEP) store_moment4(M, row, c, m, before);
             else st_elem4<BF>(M.m, (int64_t)row * M.cols + c, m);
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int row = tm.row(rr, lane + 64 * e), c = tm.col(lane + 64 * e);
                 if (row >= M.rows || c >= M.cols) continue;
-                if constexpr (BF && !KEEP) store_moment(M, row, c, mv[rr][e]);
+                if constexpr (BF && !KEEP) store_moment(M, row, c, mv[rr][e], before[e]);
                 else if constexpr (BF) st_elem<true>(M.m, (int64_t)row * M.cols + c, mv[rr][e]);
                 else stg_nt<float>(M.m + (int64_t)row * M.cols + c, mv[rr][e]);
             }

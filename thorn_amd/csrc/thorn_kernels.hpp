@@ -18,33 +18,29 @@ __device__ __forceinline__ float cautious_step(float p, float u, float lr, float
     return fmaf(u, -lr, p);
 }
 
-// This step's moment of a bf16 matrix: stored rounded into m, with the rounding residual at the same
-// place of xa (row stride ldx), from where moment_of restores it.
-__device__ __forceinline__ void store_moment(const OrthoMat& M, int row, int c, float m) {
-    const unsigned short h = bf16_round(m);
-    stg<unsigned short>(reinterpret_cast<unsigned short*>(M.m) + int64_t(row) * M.cols + c, h);
-    stg<short>(reinterpret_cast<short*>(M.xa) + int64_t(row) * M.ldx + c, bf16_residual(m, h));
+// This step's moment of a bf16 matrix: stored rounded into m, and the moment `before` it at the same
+// place of xa (row stride ldx), from which u_of makes the unrounded one again: 16 bits that lose nothing
+// (what the rounding took off has no exact form in 16 bits: of a tie it is 2^15 units up or down).
+__device__ __forceinline__ void store_moment(const OrthoMat& M, int row, int c, float m, float before) {
+    stg<unsigned short>(reinterpret_cast<unsigned short*>(M.m) + int64_t(row) * M.cols + c, bf16_round(m));
+    stg<unsigned short>(reinterpret_cast<unsigned short*>(M.xa) + int64_t(row) * M.ldx + c, bf16_of(before));
 }
-__device__ __forceinline__ void store_moment4(const OrthoMat& M, int row, int c, const float4& m) {
-    const ushort4v h{bf16_round(m.x), bf16_round(m.y), bf16_round(m.z), bf16_round(m.w)};
-    typedef short short4r __attribute__((ext_vector_type(4)));
-    stg_nt<ushort4v>(reinterpret_cast<unsigned short*>(M.m) + int64_t(row) * M.cols + c, h);
-    stg<short4r>(reinterpret_cast<short*>(M.xa) + int64_t(row) * M.ldx + c,
-                 short4r{bf16_residual(m.x, h[0]), bf16_residual(m.y, h[1]), bf16_residual(m.z, h[2]),
-                         bf16_residual(m.w, h[3])});
+__device__ __forceinline__ void store_moment4(const OrthoMat& M, int row, int c, const float4& m,
+                                              const float (&before)[4]) {
+    stg_nt<ushort4v>(reinterpret_cast<unsigned short*>(M.m) + int64_t(row) * M.cols + c,
+                     ushort4v{bf16_round(m.x), bf16_round(m.y), bf16_round(m.z), bf16_round(m.w)});
+    stg<ushort4v>(reinterpret_cast<unsigned short*>(M.xa) + int64_t(row) * M.ldx + c,
+                  ushort4v{bf16_of(before[0]), bf16_of(before[1]), bf16_of(before[2]), bf16_of(before[3])});
 }
 
-// u = g + beta1 * m of an element from the gradient and this step's updated moment.
+// u = g + beta1 * m of an element from the gradient and this step's updated moment: fp32 m as stored,
+// bf16 m made again from the moment before the step, with the arithmetic that made it (two roundings).
 template <bool BF>
 __device__ __forceinline__ float u_of(const OrthoMat& M, int row, int c, float beta1) {
     const int64_t i = int64_t(row) * M.cols + c;
-    float m;
-    if constexpr (BF)
-        m = bf16_restore(ldg<unsigned short>(reinterpret_cast<const unsigned short*>(M.m) + i),
-                         ldg<short>(reinterpret_cast<const short*>(M.xa) + int64_t(row) * M.ldx + c));
-    else
-        m = ldg<float>(M.m + i);
-    return fmaf(m, beta1, ld_elem<BF>(M.g, i));
+    const float g = ld_elem<BF>(M.g, i);
+    if constexpr (BF) return fmaf(ld_elem<true>(M.xa, int64_t(row) * M.ldx + c) * beta1 + g, beta1, g);
+    else return fmaf(ldg<float>(M.m + i), beta1, g);
 }
 template <bool BF>
 __device__ __forceinline__ float4 u_of4(const OrthoMat& M, int row, int c, float beta1) {
@@ -52,11 +48,8 @@ __device__ __forceinline__ float4 u_of4(const OrthoMat& M, int row, int c, float
     const float4 g = ld_elem4<BF, false>(M.g, i);
     float4 m;
     if constexpr (BF) {
-        typedef short short4r __attribute__((ext_vector_type(4)));
-        const ushort4v h = ldg<ushort4v>(reinterpret_cast<const unsigned short*>(M.m) + i);
-        const short4r r = ldg<short4r>(reinterpret_cast<const short*>(M.xa) + int64_t(row) * M.ldx + c);
-        m = make_float4(bf16_restore(h[0], r[0]), bf16_restore(h[1], r[1]), bf16_restore(h[2], r[2]),
-                        bf16_restore(h[3], r[3]));
+        m = ld_elem4<true, false>(M.xa, int64_t(row) * M.ldx + c);
+        m = make_float4(m.x * beta1 + g.x, m.y * beta1 + g.y, m.z * beta1 + g.z, m.w * beta1 + g.w);
     } else {
         m = ldg<float4>(M.m + i);
     }
