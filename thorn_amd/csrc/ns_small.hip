@@ -354,19 +354,21 @@ constexpr int kKeepRounds = 3;
 // -------------------------------------------------------------------------------------------------
 // Thin matrices: short side s <= 128. A workgroup's LDS holds R, Z and Q (s x s, row-major, 16 bytes of
 // padding per row) and its columns of the iterate, so between the first iterate and u' nothing goes
-// through memory but a cluster's Gram sums: every member runs the whole chain of s x s products itself,
-// the same one in each, and member i owns the 32-column blocks [nb0, nb1) of the iterate, whose Gram
-// matrix sums fp32 partial products over the members in order and whose update Q X needs no other
-// member's columns. A cluster meets at its Gram matrices and at the end, not at each of the 18
-// operations. Bound by latency: a product of two s x s matrices takes 0.6 us (s <= 32) to 2 us (s = 128)
-// against 7-8 with both operands and the result in the L2, a Gram matrix of 16 x 3072 2.4-2.9 us against 30
-// (one wave walked it), its update 3.7 against 60 (two of 16 waves, through both orientations in memory); 224 adapters of rank 16
-// 580 us in all before, 70 now.
+// through memory but a cluster's Gram matrices: every member runs the whole chain of s x s products itself,
+// the same one in each, and member i owns the 32-column blocks [nb0, nb1) of the iterate, whose update Q X
+// needs no other member's columns. A Gram matrix's elements are one MFMA chain over K each, as in the
+// schedule through the L2 (partial sums of the members' columns would give other last bits): the members of a
+// cluster deal its 32 x 32 tiles among them (thin_gram). A cluster meets at its Gram matrices and at the end,
+// not at each of the 18 operations. Bound by latency: a product
+// of two s x s matrices takes 0.6 us (s <= 32) to 2 us (s = 128) against 7-8 with both operands and the result in
+// the L2, a Gram matrix of 16 x 3072 6 us (192 dependent MFMAs of 64 cycles) against 30, its update 3.7 against 60
+// (two of 16 waves, through both orientations in memory). Step of 3072 x 16 71 us against 554, of 128 x 384 84
+// against 156; the launch over 224 adapters of rank 16 78 us against 580.
 // -------------------------------------------------------------------------------------------------
 constexpr int kThinMaxS = 128, kThinMaxCluster = 16;
 constexpr int kThinLds = 159 * 1024;
 __host__ __device__ constexpr int thin_square_bytes(int T) { return 32 * T * (64 * T + 16); }
-// the squares, or the parts of a Gram matrix that four waves share (T = 1)
+// the squares, or the ring that a cluster's Gram matrices go through
 __host__ __device__ constexpr int thin_base(int T) { return 3 * thin_square_bytes(T) > 16384 ? 3 * thin_square_bytes(T) : 16384; }
 // columns of the iterate (a multiple of 32) that fit beside them: s rows, and one of zeros for the rows
 // that pad s to 32 T
@@ -382,9 +384,6 @@ __host__ __device__ __forceinline__ int thin_cluster(int s, int l, int64_t tiles
     if (by_cols > kThinMaxCluster) return 0;
     return static_cast<int>(by_tiles < by_cols ? by_cols : by_tiles < kThinMaxCluster ? by_tiles : kThinMaxCluster);
 }
-// fp32 partial Gram matrices of a cluster, two sets (one may still be read while the next is written)
-__host__ __device__ __forceinline__ int64_t thin_partials(int64_t sp, int64_t C) { return C > 1 ? 2 * C * sp * sp : 0; }
-
 // A member's iterate columns in LDS: element (i, j), j from the member's first column, at `at(i) + 2 j`.
 struct ThinX {
     int base, ldx, s, nb0, nb1;   // bytes; 32-column blocks
@@ -458,6 +457,116 @@ __device__ __forceinline__ half4 thin_round(const floatx16& acc, int g, float al
     return h;
 }
 
+// R = X X^T of a cluster's iterate, from the workspace (slot 0) into the workspace's R: the 32 x 32 tiles on and
+// above the diagonal dealt over the members, then over a member's waves, the panel rows that they need streamed
+// by all waves through a ring of stages of 64 columns in the place of the squares (A and B are one panel), one
+// barrier a stage, a stage's fragments read while the one before it is multiplied. Ends with this wave's stores
+// issued. Bound by the chain of dependent MFMAs, 64 cycles each: 0.2 us a
+// stage; the step of 108 x 3711 (15 members) 136 us, of 16 x 60000 464, against 893 and 3370 through the L2.
+template <int T>
+__device__ __forceinline__ void thin_gram(const OrthoMat& M, const SmallView& V, int member, int C, char* lds) {
+    constexpr int SP = 32 * T, STAGE = 128 * SP, MAX = thin_base(T) / STAGE, S = MAX < 6 ? MAX : 6, TRI = T * (T + 1) / 2;
+    static_assert(S >= 3 && 4 * T <= kSmallWaves && TRI <= kSmallWaves, "ring, loads, tiles");
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    unsigned need = 0;   // 32-row blocks
+    int ti = 0, tj = 0;
+    bool has = false;
+    for (int k = member, w = 0; k < TRI; k += C, ++w) {
+        int i, j;
+        tri_decode(k, T, i, j);
+        need |= 1u << i | 1u << j;
+        if (w == wave) has = true, ti = 32 * i, tj = 32 * j;
+    }
+    if (need == 0) return;
+    // this wave's piece of a stage: 16 rows of one of its two chunks of 32 columns
+    const int chunk = wave / (2 * T), r0 = 16 * (wave % (2 * T)), r = r0 + (lane >> 2);
+    const bool loads = wave < 4 * T && (need >> (r0 / 32) & 1u);
+    const char* const src = reinterpret_cast<const char*>(V.xw(0) + int64_t(r) * V.lp + 32 * chunk) +
+                            16 * ((lane & 3) ^ ((r >> 2) & 3));
+    const uint32_t to = __builtin_amdgcn_readfirstlane(lds_address(lds)) + chunk * (64 * SP) + 64 * r0;
+    // Loads past the end read zeros, so that every stage has as many and the waits are constants.
+    const void* const zero = M.zero;
+    const int width = r < M.s ? V.lp - 32 * chunk : 0;   // (the rows that pad s: zeros)
+    int col = 0;
+    auto issue = [&](int at) {   // the next stage, into the place at byte `at`
+        if (loads) {
+            const void* p = col < width ? static_cast<const void*>(src + 2 * int64_t(col)) : zero;
+            asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"((const THORN_GLOBAL void*)p), "{m0}"(to + at)
+                         : "memory");
+        }
+        col += 64;
+    };
+    half8 a[2][4], b[2][4];
+    auto fetch = [&](int s, int at) {   // this wave's fragments of the stage there
+        if (!has) return;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            a[s][i] = frag<128, true>(lds + at + i / 2 * (64 * SP), ti, i % 2, lane);
+            b[s][i] = frag<128, true>(lds + at + i / 2 * (64 * SP), tj, i % 2, lane);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    floatx16 acc = {};
+    int at = 0;   // of the stage that is multiplied, then refilled
+    auto step = [&](int s, int k0) {   // columns k0 .. k0 + 63
+        // the next stage has landed, and every wave has this one in registers
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(S - 2) : "memory");
+        issue(at);
+        at = at == (S - 1) * STAGE ? 0 : at + STAGE;
+        fetch(s ^ 1, at);
+        if (!has || k0 >= V.lp) return;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(b[s][i], a[s][i], acc, 0, 0, 0);
+        if (k0 + 32 >= V.lp) return;
+#pragma unroll
+        for (int i = 2; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(b[s][i], a[s][i], acc, 0, 0, 0);
+    };
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");   // the squares are free; counts start at 0
+#pragma unroll
+    for (int k = 0; k < S; ++k) issue(k * STAGE);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(S - 1) : "memory");
+    fetch(0, 0);
+    for (int k0 = 0; k0 < V.lp; k0 += 128) {
+        step(0, k0);
+        step(1, k0 + 64);
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    if (!has) return;
+    _Float16* const R = V.sq(kBufR);
+    const int lr = lane & 31, lc = 4 * (lane >> 5);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const half4 h = thin_round<false>(acc, g, 1.f, 0.f, half4{});
+        stg<half4>(R + (ti + lr) * SP + tj + 8 * g + lc, h);
+        if (ti == tj) continue;   // (a diagonal tile is symmetric as computed)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) stg<_Float16>(R + (tj + 8 * g + lc + e) * SP + ti + lr, h[e]);
+    }
+}
+
+// Sum of the squares of 32 consecutive elements in order, as the schedule through the L2 adds them: lane l of the
+// lower half of the wave holds elements 8 g + 0 .. 3 in h[g], lane l + 32 elements 8 g + 4 .. 7; both get it.
+__device__ __forceinline__ float thin_sum_squares(const half4 (&h)[4]) {
+    float t = 0.f;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {   // (what the other half of the wave adds meanwhile is dropped)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float f = static_cast<float>(h[g][e]);
+                t += f * f;
+            }
+            // low, high: the value of the wave's lower and upper half in both (the builtin's second result comes
+            // back as its first with this compiler)
+            float low = t, high = t;
+            asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(low), "+v"(high));
+            t = half == 0 ? low : high;
+        }
+    }
+    return t;
+}
+
 // The schedule of one matrix with s_p = 32 T, its first iterate in LDS. Accumulators are transposed
 // products (B^T A^T): lane l has row (l & 31) of a 32 x 32 tile, columns 8 g + 4 (l / 32) + 0..3 in
 // registers 4 g + 0..3.
@@ -465,17 +574,13 @@ template <int T>
 __device__ __forceinline__ void thin_schedule(const OrthoMat& M, const SmallView& V, const SmallOp* ops, int nops,
                                               int member, int C, char* lds, SmallSync& sync, unsigned tslot) {
     constexpr int SP = 32 * T, LDQ = 2 * SP + 16, SQ = thin_square_bytes(T), TILES = T * T;
-    constexpr int SPLIT = T == 1 ? 4 : 1;   // waves that share a Gram tile's contraction
-    static_assert(TILES * SPLIT <= kSmallWaves && SPLIT * 4096 <= thin_base(1), "waves, LDS");
+    static_assert(TILES <= kSmallWaves, "a wave per tile");
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_address(lds));
     const ThinX X(M, V, member, C);
-    // this wave's tile of an s x s product, and its part of a Gram matrix's contraction
-    const int tile = wave % TILES, part = wave / TILES;
-    const int ti = 32 * (tile / T), tj = 32 * (tile % T);
+    // this wave's tile of an s x s product
+    const int ti = 32 * (wave % TILES / T), tj = 32 * (wave % T);
     const bool has = wave < TILES;
-    float* const parts = reinterpret_cast<float*>(V.base + 8 * V.sqe + 4 * V.xe);
-    int grams = 0;
     // Where each of R, Z, QA, QB is (a byte each: an array indexed by the operation would go to memory).
     // A product replaces its C term in place (R Z is made from R, and the next R from R Z; Q from Q), but
     // Z has a place of its own, and a Q that starts anew another.
@@ -493,45 +598,40 @@ __device__ __forceinline__ void thin_schedule(const OrthoMat& M, const SmallView
         const int kr = 8 * (lane >> 5) + ((lane & 15) >> 2);   // k row of a transposing read
         ts_op(tslot, q, 0);
         if (op.kind == kOpGram) {
-            floatx16 acc = {};
-            if (part < SPLIT) {
-                const int ra = X.at(ti + lr), rb = X.at(tj + lr), nks = 2 * (X.nb1 - X.nb0);
-#pragma unroll 4
-                for (int ks = part; ks < nks; ks += SPLIT)
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(thin_row_frag(lds, rb, ks, lane),
-                                                                 thin_row_frag(lds, ra, ks, lane), acc, 0, 0, 0);
-            }
             move(kBufR, 0);
-            if constexpr (SPLIT > 1) {   // the parts, summed in order into the first wave's
-                float* const red = reinterpret_cast<float*>(lds);
-                if (part > 0 && part < SPLIT) {
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) red[part * 1024 + 64 * r + lane] = acc[r];
-                }
-                __syncthreads();
-                if (part == 0) {
-#pragma unroll
-                    for (int p = 1; p < SPLIT; ++p)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) acc[r] += red[p * 1024 + 64 * r + lane];
-                }
-                __syncthreads();   // read before R replaces them
-            }
-            if (C > 1) {   // the members' sums, in order
-                float* const set = parts + int64_t(grams++ & 1) * C * SP * SP;
-                if (has) {
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) stg<float>(set + (member * TILES + tile) * 1024 + 64 * r + lane, acc[r]);
-                }
+            if (C > 1) {
+                if (q > 0) sync.wait();   // every member's columns of the iterate (the first one's are there)
+                thin_gram<T>(M, V, member, C, lds);
                 sync.wait();
-                if (has) {
-                    acc = floatx16{};
-                    for (int m = 0; m < C; ++m)
+                constexpr int PER = SP / 8;   // 16-byte chunks of a row
+                for (int k = tid; k < SP * PER; k += kSmallThreads)
+                    *reinterpret_cast<half8*>(lds + k / PER * LDQ + 16 * (k % PER)) = ldg<half8>(V.sq(kBufR) + 8 * k);
+            } else if (has) {
+                floatx16 acc = {};
+                const int ra = X.at(ti + lr), rb = X.at(tj + lr), nks = 2 * (X.nb1 - X.nb0);
+                // four steps of 16 columns are read while the four before them are multiplied
+                half8 a[2][4], b[2][4];
+                auto fetch = [&](int s, int k0) {
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) acc[r] += ldg<float>(set + (m * TILES + tile) * 1024 + 64 * r + lane);
+                    for (int i = 0; i < 4; ++i) {
+                        const int ks = min(k0 + i, nks - 1);
+                        a[s][i] = thin_row_frag(lds, ra, ks, lane);
+                        b[s][i] = thin_row_frag(lds, rb, ks, lane);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                };
+                auto multiply = [&](int s, int k0) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (k0 + i < nks) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(b[s][i], a[s][i], acc, 0, 0, 0);
+                };
+                fetch(0, 0);
+                for (int k0 = 0; k0 < nks; k0 += 8) {
+                    fetch(1, k0 + 4);
+                    multiply(0, k0);
+                    fetch(0, k0 + 8);
+                    multiply(1, k0 + 4);
                 }
-            }
-            if (has) {
 #pragma unroll
                 for (int g = 0; g < 4; ++g)
                     *reinterpret_cast<half4*>(lds + (ti + lr) * LDQ + 2 * (tj + 8 * g + lc)) =
@@ -588,19 +688,21 @@ __device__ __forceinline__ void thin_schedule(const OrthoMat& M, const SmallView
 #pragma unroll
                         for (int ks = 0; ks < 2 * T; ++ks)
                             acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[ks], thin_row_frag(lds, Q + row * LDQ, ks, lane), acc, 0, 0, 0);
-                        float sq = 0.f;
+                        half4 h[4];
 #pragma unroll
                         for (int g = 0; g < 4; ++g) {
-                            half4* const px = reinterpret_cast<half4*>(lds + X.at(row) + 2 * (j0 + 8 * g + lc));
-                            const half4 h = op.c >= 0 ? thin_round<true>(acc, g, 1.f, op.beta, *px)
-                                                      : thin_round<false>(acc, g, 1.f, 0.f, half4{});
-                            if (row < M.s && !op.fin) *px = h;
-                            if (row < M.s && op.fin) stg<half4>(M.xa + int64_t(row) * M.ldx + n0 + 8 * g + lc, h);
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) sq += static_cast<float>(h[e]) * static_cast<float>(h[e]);
+                            const int c = 8 * g + lc;
+                            half4* const px = reinterpret_cast<half4*>(lds + X.at(row) + 2 * (j0 + c));
+                            h[g] = op.c >= 0 ? thin_round<true>(acc, g, 1.f, op.beta, *px)
+                                             : thin_round<false>(acc, g, 1.f, 0.f, half4{});
+                            if (row >= M.s) continue;
+                            if (op.fin) stg<half4>(M.xa + int64_t(row) * M.ldx + n0 + c, h[g]);
+                            else *px = h[g];
+                            // for the cluster's next Gram matrix (its last one's readers have met since)
+                            if (!op.fin && C > 1) stg<half4>(V.xw(0) + int64_t(row) * V.lp + n0 + c, h[g]);
                         }
                         if (op.fin && (M.flags & kFlagPNN)) {
-                            sq += __shfl_xor(sq, 32);
+                            const float sq = thin_sum_squares(h);
                             if (lane < 32 && row < M.s) M.rowsqpart[int64_t(n0 >> 5) * M.rows + row] = sq;
                         }
                     }
@@ -615,16 +717,14 @@ __device__ __forceinline__ void thin_schedule(const OrthoMat& M, const SmallView
                         for (int ks = 0; ks < 2 * T; ++ks)
                             acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(thin_row_frag(lds, Q + (32 * t + lr) * LDQ, ks, lane), x[ks],
                                                                          acc, 0, 0, 0);
-                        float sq = 0.f;
+                        half4 h[4];
 #pragma unroll
                         for (int g = 0; g < 4; ++g) {   // (a tall matrix is not square: no beta X)
-                            const half4 h = thin_round<false>(acc, g, 1.f, 0.f, half4{});
-                            if (row < M.rows) stg<half4>(M.xa + int64_t(row) * M.ldx + 32 * t + 8 * g + lc, h);
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) sq += static_cast<float>(h[e]) * static_cast<float>(h[e]);
+                            h[g] = thin_round<false>(acc, g, 1.f, 0.f, half4{});
+                            if (row < M.rows) stg<half4>(M.xa + int64_t(row) * M.ldx + 32 * t + 8 * g + lc, h[g]);
                         }
                         if (M.flags & kFlagPNN) {
-                            sq += __shfl_xor(sq, 32);
+                            const float sq = thin_sum_squares(h);
                             if (lane < 32 && row < M.rows) M.rowsqpart[int64_t(t) * M.rows + row] = sq;
                         }
                     }
@@ -643,70 +743,6 @@ __device__ __forceinline__ void thin_schedule(const OrthoMat& M, const SmallView
 constexpr int kQuarter = 256;
 static_assert(kSmallThreads == 4 * kQuarter, "four quarters of a workgroup");
 
-// ortho_pre_kernel's momentum for a matrix without decouple_md, Magma or an Adam step, on
-// elementwise tile t by one quarter (t256 = 0..255 in that kernel's thread layout): m <- beta1 m +
-// g, stored; returns this thread's sum of u^2, u = g + beta1 m, in that kernel's order.
-// KEEP: u of this thread's elements into u[4 rr + e] (0 outside the matrix), for small_x0_tile, which
-// then needs neither the gradient nor the moment again.
-template <bool BF, bool KEEP>
-__device__ __forceinline__ float small_momentum_tile(const OrthoMat& M, int t, int t256, float (&u)[16]) {
-    const int lane = t256 & 63, wave = t256 >> 6;
-    const TileMap tm(M, t, wave);
-    const float beta1 = M.beta1;
-    const bool vec = M.flags & kFlagVec4;
-    float gv[4][4], mv[4][4];   // loads first
-#pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-        if (vec) {
-            const int row = tm.row(rr, 4 * lane), c = tm.col(4 * lane);
-            float4 g = make_float4(0.f, 0.f, 0.f, 0.f), m = g;
-            if (row < M.rows && c < M.cols) {
-                g = ld_elem4<BF>(M.g, (int64_t)row * M.cols + c);
-                m = ld_elem4<BF>(M.m, (int64_t)row * M.cols + c);
-            }
-            gv[rr][0] = g.x; gv[rr][1] = g.y; gv[rr][2] = g.z; gv[rr][3] = g.w;
-            mv[rr][0] = m.x; mv[rr][1] = m.y; mv[rr][2] = m.z; mv[rr][3] = m.w;
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int row = tm.row(rr, lane + 64 * e), c = tm.col(lane + 64 * e);
-                const bool ok = row < M.rows && c < M.cols;
-                gv[rr][e] = ok ? ld_elem<BF>(M.g, (int64_t)row * M.cols + c) : 0.f;
-                mv[rr][e] = ok ? ld_elem<BF>(M.m, (int64_t)row * M.cols + c) : 0.f;
-            }
-        }
-    }
-    float nrm = 0.f;
-#pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-        [[maybe_unused]] const float before[4] = {mv[rr][0], mv[rr][1], mv[rr][2], mv[rr][3]};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            mv[rr][e] = mv[rr][e] * beta1 + gv[rr][e];
-            const float x = fmaf(mv[rr][e], beta1, gv[rr][e]);
-            nrm += x * x;   // (zeros outside the matrix)
-            if constexpr (KEEP) u[4 * rr + e] = x;
-        }
-        if (vec) {
-            const int row = tm.row(rr, 4 * lane), c = tm.col(4 * lane);
-            if (row >= M.rows || c >= M.cols) continue;
-            const float4 m = make_float4(mv[rr][0], mv[rr][1], mv[rr][2], mv[rr][3]);
-            if constexpr (BF && !KEEP) store_moment4(M, row, c, m, before);
-            else st_elem4<BF>(M.m, (int64_t)row * M.cols + c, m);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int row = tm.row(rr, lane + 64 * e), c = tm.col(lane + 64 * e);
-                if (row >= M.rows || c >= M.cols) continue;
-                if constexpr (BF && !KEEP) store_moment(M, row, c, mv[rr][e], before[e]);
-                else if constexpr (BF) st_elem<true>(M.m, (int64_t)row * M.cols + c, mv[rr][e]);
-                else stg_nt<float>(M.m + (int64_t)row * M.cols + c, mv[rr][e]);
-            }
-        }
-    }
-    return nrm;
-}
-
 // First iterate of elementwise tile t by one quarter: the values of small_x0; the orientation in which
 // the tile's columns are contiguous stored directly, the other through the quarter's LDS transpose `tt`
 // (a row per column of the tile, holding its R = 4096 / 2^lw rows, R + 8 halves apart) as 16-byte chunks
@@ -714,13 +750,12 @@ __device__ __forceinline__ float small_momentum_tile(const OrthoMat& M, int t, i
 // number of times (block barriers); `active`: t is a tile of the matrix.
 constexpr int kX0Halves = 256 * 24;   // the largest transpose: 256 columns of 16 rows
 static_assert(4 * kX0Halves * 2 <= kSmallStages * kSmallStageBytes, "four transposes in the ring");
-// KEEP: u as small_momentum_tile kept it.
+// KEEP: u as momentum_tile gave it.
 template <bool BF, bool KEEP>
 __device__ __forceinline__ void small_x0_tile(const OrthoMat& M, const SmallView& V, int t, int t256, bool active,
                                               float denom, _Float16* tt, const float (&u)[16]) {
-    const int lane = t256 & 63, wave = t256 >> 6;
-    const TileMap tm(M, t, wave);
-    const int R = 4096 >> tm.lw, pitch = R + 8, rt0 = t / M.mom_tiles_c * R;   // the tile's rows
+    const TileMap tm(M, t, t256);
+    const int R = 4096 >> tm.lw, pitch = R + 8;   // the tile's rows
     _Float16* const direct = M.tall ? V.xwt(0) : V.xw(0);   // row r of the parameter, contiguous
     const int ldd = M.tall ? V.sp : V.lp;
     _Float16* const tpose = M.tall ? V.xw(0) : V.xwt(0);    // column c of the parameter, contiguous
@@ -729,17 +764,14 @@ __device__ __forceinline__ void small_x0_tile(const OrthoMat& M, const SmallView
         const float beta1 = M.beta1;
         const bool vec = KEEP && (M.flags & kFlagVec4);     // the elements that u belongs to
 #pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int i = vec ? 4 * lane + e : lane + 64 * e, r = tm.row(rr, i), c = tm.col(i);
-                _Float16 x = _Float16(0.f);
-                if (r < M.rows && c < M.cols) {
-                    x = (_Float16)((KEEP ? u[4 * rr + e] : u_of<BF>(M, r, c, beta1)) / denom);
-                    direct[int64_t(r) * ldd + c] = x;
-                }
-                tt[(c - tm.c0) * pitch + r - rt0] = x;
+        for (int k = 0; k < 16; ++k) {
+            const int r = vec ? tm.vrow(k / 4) : tm.erow(k), c = vec ? tm.vcol() + k % 4 : tm.ecol(k);
+            _Float16 x = _Float16(0.f);
+            if (r < M.rows && c < M.cols) {
+                x = (_Float16)((KEEP ? u[k] : u_of<BF>(M, r, c, beta1)) / denom);
+                direct[int64_t(r) * ldd + c] = x;
             }
+            tt[(c - tm.c0) * pitch + r - tm.row0] = x;
         }
     }
     lds_barrier();   // (not the stores)
@@ -748,16 +780,16 @@ __device__ __forceinline__ void small_x0_tile(const OrthoMat& M, const SmallView
 #pragma unroll
         for (int h2 = 0; h2 < 2; ++h2) {
             const int chunk = t256 + kQuarter * h2, cl = chunk / per, h = chunk % per;
-            if (tm.c0 + cl < M.cols && rt0 + 8 * h < ldt)
-                stg<half8>(tpose + int64_t(tm.c0 + cl) * ldt + rt0 + 8 * h,
+            if (tm.c0 + cl < M.cols && tm.row0 + 8 * h < ldt)
+                stg<half8>(tpose + int64_t(tm.c0 + cl) * ldt + tm.row0 + 8 * h,
                            *reinterpret_cast<const half8*>(tt + cl * pitch + 8 * h));
         }
     }
     lds_barrier();   // the transpose is read before the next round writes it
 }
 
-// Before the schedule: the momentum and the tile partials of ||u||^2 (each tile's sum over its 256
-// threads as block_sum adds them), a cluster barrier, the norm and, in member 0, the matrix's
+// Before the schedule: the momentum and the tile partials of ||u||^2 (momentum_tile, as
+// ortho_pre_kernel makes them), a cluster barrier, the norm and, in member 0, the matrix's
 // scalars, the first iterate f16(u / (||u|| + 1e-8)) and its padding, a cluster barrier.
 // A thin matrix of one workgroup leaves its first iterate in LDS; returns whether it did.
 template <bool BF, bool KEEP>
@@ -766,20 +798,14 @@ __device__ __forceinline__ bool small_fused_prologue_as(const OrthoMat& M, const
     const int q = threadIdx.x / kQuarter, t256 = threadIdx.x % kQuarter;
     const int ntiles = M.mom_tiles_r * M.mom_tiles_c, per = 4 * C;
     float u[KEEP ? kKeepRounds : 1][16];
+    float* const quads = reinterpret_cast<float*>(stages) + 64 * q;
     auto norm_round = [&](int t0, float (&ur)[16]) {
         const int t = t0 + 4 * member + q;
-        float nrm = t < ntiles ? small_momentum_tile<BF, KEEP>(M, t, t256, ur) : 0.f;
-        nrm = wave_sum(nrm);
         // (barriers for LDS alone: the moments' stores drain behind them; 4 us a round when waited for)
-        lds_barrier();   // the previous round's reads of red are done
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = nrm;
+        lds_barrier();   // the previous round's quads are read
+        if (t < ntiles) momentum_tile<BF, !KEEP>(M, t, t256, false, ur, quads);
         lds_barrier();
-        if (t < ntiles && t256 == 0) {
-            float sum = 0.f;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sum += red[4 * q + i];
-            M.normpart[t] = sum;
-        }
+        if (t < ntiles) tile_partials(M, t, t256, false, quads);
     };
     // (the same trip count in every quarter: barriers)
     if constexpr (KEEP) {
@@ -802,12 +828,11 @@ __device__ __forceinline__ bool small_fused_prologue_as(const OrthoMat& M, const
             for (int r = 0; r < kKeepRounds; ++r) {
                 const int t = r * per + q;
                 if (t >= ntiles) continue;
-                const TileMap tm(M, t, t256 >> 6);
+                const TileMap tm(M, t, t256);
                 const bool vec = M.flags & kFlagVec4;
 #pragma unroll
                 for (int k = 0; k < 16; ++k) {
-                    const int i = vec ? 4 * (t256 & 63) + k % 4 : (t256 & 63) + 64 * (k % 4);
-                    const int row = tm.row(k / 4, i), c = tm.col(i);
+                    const int row = vec ? tm.vrow(k / 4) : tm.erow(k), c = vec ? tm.vcol() + k % 4 : tm.ecol(k);
                     if (row >= M.rows || c >= M.cols) continue;
                     *reinterpret_cast<_Float16*>(stages + X.at(M.tall ? c : row) + 2 * (M.tall ? row : c)) =
                         (_Float16)(u[r][k] / denom);
@@ -817,7 +842,10 @@ __device__ __forceinline__ bool small_fused_prologue_as(const OrthoMat& M, const
             return true;
         }
     }
-    if (member == 0 && !thin) small_x0_padding(M, V, threadIdx.x, kSmallThreads);   // (thin_clear does that)
+    if (member == 0 && !thin) small_x0_padding(M, V, threadIdx.x, kSmallThreads);
+    if (member == 0 && thin && M.l < V.lp)   // (what thin_gram reads of it)
+        for (int e = threadIdx.x; e < M.s * (V.lp - M.l); e += kSmallThreads)
+            V.xw(0)[int64_t(e / (V.lp - M.l)) * V.lp + M.l + e % (V.lp - M.l)] = _Float16(0.f);
     _Float16* const tt = reinterpret_cast<_Float16*>(stages) + q * kX0Halves;
     auto x0_round = [&](int t0, const float (&ur)[16]) {
         const int t = t0 + 4 * member + q;

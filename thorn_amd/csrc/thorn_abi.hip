@@ -735,8 +735,7 @@ int thorn_ortho_plan_create(const ThornOrthoMatDesc* descs, int n, thorn_ortho_p
         const bool square = L.rows == L.cols;   // the plain quintic needs no Q (thorn.py:654-658)
         if (L.is_small) {
             const size_t sp = align_up(L.s, 32), lp = align_up(L.l, 32);
-            L.small = take((8 * sp * sp + 4 * sp * lp) * 2 +
-                           (L.thin ? thorn::thin_partials(sp, L.cluster) * sizeof(float) : 0));
+            L.small = take((8 * sp * sp + 4 * sp * lp) * 2);
             L.small_bar = take(thorn::kSmallBarWords * sizeof(int));
         } else {
             L.small = L.small_bar = kNone;
@@ -748,14 +747,14 @@ int thorn_ortho_plan_create(const ThornOrthoMatDesc* descs, int n, thorn_ortho_p
         L.qa = square ? kNone : take(sbytes);
         L.qb = square ? kNone : take(sbytes);
         L.rowpsq = L.norm_rows ? take(sizeof(float) * size_t(L.mom_tiles_c) * L.rows) : kNone;
-        L.normpart = take(sizeof(float) * mom_tiles);
+        L.normpart = take(sizeof(float) * thorn::norm_tiles(L.rows, L.cols));
         L.rowpart = md ? take(sizeof(float) * size_t(L.mom_tiles_c) * L.rows) : kNone;
         L.colpart = (L.flags & THORN_MAT_MD) ? take(sizeof(float) * size_t(L.mom_tiles_r) * L.cols) : kNone;
         L.rowsqpart = pnn ? take(sizeof(float) * size_t(L.rowsq_tiles) * L.rows) : kNone;
         L.rowscale = pnn || L.norm_rows ? take(sizeof(float) * L.rows) : kNone;
         L.scal = take(sizeof(float) * 8);
         L.psqpart = md ? take(sizeof(float) * L.n_psq) : kNone;
-        L.magpart = take(sizeof(float4) * mom_tiles);
+        L.magpart = take(sizeof(float4) * thorn::norm_tiles(L.rows, L.cols));
         plan->mats.push_back(L);
     }
     plan->ws_bytes = std::max<size_t>(ws, kAlign);
