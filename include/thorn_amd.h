@@ -264,8 +264,10 @@ int thorn_adam_sparse_step(const ThornAdamSparseStep* step, void* stream);
  * A, B and C are read where they are when their chunks of 8 elements are aligned (a unit stride, the
  * other strides and the length along the unit stride multiples of 8, 16-byte aligned pointers; C
  * with contiguous rows; not an A whose columns are contiguous beside a B whose columns are), and
- * through copies in the workspace otherwise. workspace: thorn_sym_addmm_workspace_needed() bytes of
- * device memory for these very tensors (0: it may be null), at most thorn_sym_addmm_workspace_bytes(),
+ * through copies in the workspace otherwise. out may share memory with them: C may be out itself, and
+ * any other operand whose bytes overlap out's is read through a copy too. workspace:
+ * thorn_sym_addmm_workspace_needed() bytes of device memory for these very tensors beside an out that
+ * shares nothing with them (0: it may be null), thorn_sym_addmm_workspace_bytes() for any out,
  * 256-byte aligned; calls that share it must not overlap. Limits: nn <= 65535 (thorn.py:332), m * round_up(k, 32) and
  * m * round_up(m, 8) below 2^30 elements.
  * ------------------------------------------------------------------------------------------ */

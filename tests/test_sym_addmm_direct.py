@@ -105,3 +105,52 @@ def test_in_place_reads_nothing_behind_the_operand():
     want = torch.ops.thorn.sym_addmm(v, v.mT.contiguous(), None, 1.0, 0.0)
     for a, b in ((x, x.mT), (x, xt), (xt.mT, xt)):
         assert torch.equal(torch.ops.thorn.sym_addmm(a, b, None, 1.0, 0.0), want)
+
+
+def _call(lib, a, sa, b, sb, c, sc, c_mats, out, shape, beta, ws, nbytes, stream=None):
+    i3 = lambda s: (ctypes.c_int64 * 3)(*s)
+    return lib.thorn_sym_addmm(a, i3(sa), b, i3(sb), c, i3(sc) if c else None, c_mats, out, *shape, 1.0, beta, ws, nbytes,
+                               stream)
+
+
+def test_out_over_an_operand_needs_its_copy():
+    """Operands that could be read in place, beside an out that shares memory with one of them: refused without
+    the workspace for its copy (on the host, before anything is launched)."""
+    lib = _lib.load()
+    nn, m = 2, 256
+    mat = (m * m, m, 1)
+    size = 2 * nn * m * m
+    a, b, c = (size * i for i in range(1, 4))
+    for sc, c_mats, out in ((None, 0, a), (None, 0, a - 16), (None, 0, a + size - 16), (None, 0, b + size // 2), (mat, nn, b),
+                            (mat, nn, c + size // 2),                     # a matrix off C
+                            ((0, m, 1), 1, c),                            # one C for two products
+                            ((2 * m * m, m, 1), nn, c)):                  # C of other strides
+        rc = _call(lib, a, mat, b, mat, c if sc else None, sc, c_mats, out, (nn, m, m), 1.0, None, 0)
+        assert rc != 0 and 'workspace' in lib.thorn_last_error().decode(), (sc, c_mats, out)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('shape', [(3, 512, 512), (2, 520, 40), (1, 264, 264), (2, 250, 250)],
+                         ids=lambda s: 'x'.join(map(str, s)))
+def test_out_over_an_operand(shape):
+    nn, m, k = shape
+    print(f'[gpu] sym_addmm, out over an operand, {shape}', flush=True)
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(m + k + 1)
+    n_ab, n_out = nn * m * k, nn * m * m
+    pool = torch.randn(4 * max(n_ab, n_out) + 4096, generator=gen).half().to(DEV)
+    nbytes = lib.thorn_sym_addmm_workspace_bytes(nn, m, k, nn)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+    ab, mat = (m * k, k, 1), (m * m, m, 1)
+    for name, at_a, at_c, at_out in (('a', 0, None, 0), ('inside a', 2048, None, 0), ('across b', 0, None, n_ab // 2 // 8 * 8),
+                                     ('c', 0, n_ab, n_ab), ('c, shifted', 0, n_ab + 64, n_ab)):
+        buf = pool.clone()
+        a = buf[at_a:at_a + n_ab].view(nn, m, k)
+        c = None if at_c is None else buf[at_c:at_c + n_out].view(nn, m, m)
+        want = torch.ops.thorn.sym_addmm(a, a.mT, c, 1.0, -0.5)
+        needed = nbytes if name != 'c' or m % 8 or k % 8 else 0   # C may be out itself
+        rc = _call(lib, a.data_ptr(), ab, a.data_ptr(), (m * k, 1, k), c.data_ptr() if c is not None else None, mat,
+                   0 if c is None else nn, buf.data_ptr() + 2 * at_out, shape, -0.5, ws.data_ptr() if needed else None,
+                   needed, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, (name, lib.thorn_last_error())
+        assert torch.equal(buf[at_out:at_out + n_out].view(nn, m, m), want), name

@@ -8,6 +8,7 @@
 #include "update_kernels.hip"
 
 #include <algorithm>
+#include <array>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -568,21 +569,40 @@ bool sym_direct(const void* p, int64_t mat, int64_t line, int64_t elem, int64_t 
     return false;
 }
 
+// Whether a tensor of f16 elements (strides of its three sides, `size` long) and `bytes` from `out` on share memory,
+// by their first and last bytes.
+bool sym_overlaps(const void* t, const int64_t* strides, std::array<int64_t, 3> size, const void* out, size_t bytes) {
+    int64_t lo = 0, hi = 0;
+    for (int i = 0; i < 3; ++i) (strides[i] < 0 ? lo : hi) += strides[i] * (size[i] - 1);
+    const auto at = static_cast<int64_t>(reinterpret_cast<uintptr_t>(t)), o = static_cast<int64_t>(reinterpret_cast<uintptr_t>(out));
+    return at + 2 * lo < o + static_cast<int64_t>(bytes) && o < at + 2 * hi + 2;
+}
+
+// out: the product's result, or null where it is not known. Tiles are stored while others are still computed, so an
+// operand that shares memory with it is copied first; but C may be out itself (the same elements at the same
+// places): a tile reads C only where it stores alone, and what a mirrored tile stores is not read.
 SymAddmmLayout sym_addmm_layout(const void* a, const int64_t* as, const void* b, const int64_t* bs, const void* c,
-                                const int64_t* cs, int64_t c_mats, int64_t nn, int64_t m, int64_t k) {
+                                const int64_t* cs, int64_t c_mats, int64_t nn, int64_t m, int64_t k, const void* out) {
     SymAddmmLayout L;
     L.kp = std::max<int64_t>(32, cdiv(k, 32) * 32);
     L.mp = cdiv(m, 8) * 8;
     L.a_km = L.b_km = true;
     // b's lines are B's columns
-    bool a_ok = k > 0 && as && sym_direct(a, as[0], as[1], as[2], nn, m, k, &L.a_km);
-    const bool b_ok = k > 0 && bs && sym_direct(b, bs[0], bs[2], bs[1], nn, m, k, &L.b_km);
+    const size_t out_bytes = size_t(nn) * m * m * 2;
+    bool a_ok = k > 0 && as && sym_direct(a, as[0], as[1], as[2], nn, m, k, &L.a_km) &&
+                !(out && sym_overlaps(a, as, {nn, m, k}, out, out_bytes));
+    bool b_ok = k > 0 && bs && sym_direct(b, bs[0], bs[2], bs[1], nn, m, k, &L.b_km) &&
+                !(out && sym_overlaps(b, bs, {nn, k, m}, out, out_bytes));
+    if (!a_ok) L.a_km = true;   // a copy's
+    if (!b_ok) L.b_km = true;
     if (a_ok && !L.a_km && !(b_ok && !L.b_km)) {   // an MN-major A beside a K-major B
         a_ok = false;
         L.a_km = true;
     }
+    const bool c_out = c == out && (nn == 1 || (c_mats > 1 && cs && cs[0] == m * m));
     const bool c_ok = cs && m % 8 == 0 && cs[2] == 1 && cs[1] == m && (c_mats <= 1 || cs[0] % 8 == 0) &&
-                      (reinterpret_cast<uintptr_t>(c) & 15u) == 0;
+                      (reinterpret_cast<uintptr_t>(c) & 15u) == 0 &&
+                      (!out || c_out || !sym_overlaps(c, cs, {c_mats, m, m}, out, out_bytes));
     size_t off = 0;
     auto take = [&](size_t bytes) { const size_t o = off; off = align_up(off + bytes, kAlign); return o; };
     L.a = a_ok ? kNone : take(size_t(nn) * m * L.kp * 2);
@@ -1470,7 +1490,7 @@ int thorn_adam_sparse_step(const ThornAdamSparseStep* S, void* stream) {
 
 size_t thorn_sym_addmm_workspace_bytes(int64_t nn, int64_t m, int64_t k, int64_t c_mats) {
     if (nn < 0 || m < 0 || k < 0 || c_mats < 0) return 0;
-    return std::max<size_t>(sym_addmm_layout(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, c_mats, nn, m, k).bytes,
+    return std::max<size_t>(sym_addmm_layout(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, c_mats, nn, m, k, nullptr).bytes,
                             kAlign);
 }
 
@@ -1478,7 +1498,7 @@ size_t thorn_sym_addmm_workspace_needed(const void* a, const int64_t* as, const 
                                         const void* c, const int64_t* cs, int64_t c_mats, int64_t nn, int64_t m,
                                         int64_t k) {
     if (nn < 0 || m < 0 || k < 0 || c_mats < 0) return 0;
-    return sym_addmm_layout(a, as, b, bs, c, cs, c_mats, nn, m, k).bytes;
+    return sym_addmm_layout(a, as, b, bs, c, cs, c_mats, nn, m, k, nullptr).bytes;
 }
 
 int thorn_sym_addmm(const void* a, const int64_t* as, const void* b, const int64_t* bs, const void* c,
@@ -1491,7 +1511,7 @@ int thorn_sym_addmm(const void* a, const int64_t* as, const void* b, const int64
     if (nn == 0 || m == 0) return THORN_OK;
     if (!a || !b || !as || !bs || !out || (c_mats > 0 && (!c || !cs)))
         return fail(THORN_ERR_INVALID, "thorn_sym_addmm: null argument");
-    const SymAddmmLayout L = sym_addmm_layout(a, as, b, bs, c, cs, c_mats, nn, m, k);
+    const SymAddmmLayout L = sym_addmm_layout(a, as, b, bs, c, cs, c_mats, nn, m, k, out);
     if (m * L.kp >= (int64_t(1) << 30) || m * L.mp >= (int64_t(1) << 30))
         return fail(THORN_ERR_INVALID, "thorn_sym_addmm: a matrix of 2^30 elements or more");
     if (L.bytes > 0 && (!workspace || workspace_bytes < L.bytes || (reinterpret_cast<uintptr_t>(workspace) & (kAlign - 1)) != 0))
