@@ -3,6 +3,7 @@ copies: every kind in one group steps as it does alone, and what was refused sta
 import pytest
 import torch
 
+import thorn_amd.optim as OPT
 from thorn_amd import THORN
 
 DEV = 'cuda:0'
@@ -89,3 +90,14 @@ def test_a_mixed_group_steps_as_its_parameters_alone(orthogonalize, momentum_ali
         if not momentum_align:
             assert torch.equal(p, alone[i]), name
             assert torch.equal(opt.state[p]['moment'], opts[i].state[alone[i]]['moment']), name
+
+
+def test_release_windows_with_clusters_take_two_streams():
+    """Small-matrix launches side by side must leave an XCD's 32 CUs a place for the last member of a cluster:
+    a launch holds at most 15 for one that is not complete."""
+    small, thin, large = (torch.empty(s, device='meta') for s in ((256, 640), (3, 128, 4096), (300, 4099)))
+    streams = lambda w, orthogonalize=True: {OPT._release_stream(i, w, orthogonalize) for i in range(12)}
+    for w in ([small], [thin], [large, small], [thin, large, large]):
+        assert 15 * len(streams(w)) < 32 and streams(w) == {0, 1}
+    assert streams([large]) == streams([large, large]) == {0, 1, 2}
+    assert streams([small, thin], False) == {0, 1, 2}   # an Adam group has no clusters

@@ -805,6 +805,13 @@ CHAIN_MIN_COST = 2e10
 # Streams of the gradient-release steps (_release_step): with the caller's own, as many as the
 # device's 4 hardware queues of a process (4 of them measured 54.8 ms on config 2's hooks, 3 41.2).
 RELEASE_STREAMS = 3
+# ... and those that windows with small matrices take turns on. A cluster of the small-matrix launch holds its
+# CUs while it waits for its last member, so launches side by side must not fill an XCD (32 CUs) with clusters
+# that miss one: the blocks of an XCD start in order, so a launch has at most one such cluster there, of at most
+# 15 CUs, and two launches leave two free. With three, each of 12 members or more, every one could wait for the
+# others until the wait's limit ends the step in an error. (Chains of one step are two streams as well. Launches
+# of other optimizers or of a caller's own streams are not counted here.)
+RELEASE_CLUSTER_STREAMS = 2
 RELEASE_OVERLAP = True   # False: every released step on the caller's stream, in order
 # Gradient release keeps the dense gradients of a group's parameters until this many bytes of them
 # are there (or backward ends) and steps them as one plan or one Adam launch: one parameter's
@@ -816,6 +823,13 @@ RELEASE_WINDOW_BYTES = 256 << 20
 # chains' GEMMs (config 2 on two MI355X boxes: 6.68-6.69 against 6.75-6.77 and 6.70-6.74 against
 # 6.74-6.76 ms per step).
 ADAM_OVERLAP = True
+
+
+def _release_stream(i: int, params: list, orthogonalize: bool) -> int:
+    """The release stream of a backward pass's window number i."""
+    clusters = orthogonalize and any(min(s[:2]) <= SMALL_MAX_S and s[0] * s[1] < SMALL_MAX_ELEMS
+                                     for s in map(_matrix_view, params))
+    return i % (RELEASE_CLUSTER_STREAMS if clusters else RELEASE_STREAMS)
 
 
 def _wait_for(home: torch.cuda.Stream) -> None:
@@ -1565,7 +1579,7 @@ class THORN(Optimizer):
             return
         src, entries, _ = w
         gi, dev = key
-        k = self._release_next % RELEASE_STREAMS
+        k = _release_stream(self._release_next, [p for p, _ in entries], self.param_groups[gi]['orthogonalize'])
         self._release_next += 1
         st = self._chain_streams(dev, RELEASE_STREAMS)[k]
         evs = self._release_events.get(dev)
