@@ -57,7 +57,8 @@ enum {
                                       points at `rows` values */
 #define THORN_MAT_BF16 32          /* p, g and m are bf16; not with MD, MD_SCALAR or ADAM */
 #define THORN_MAT_TILES_128 64     /* on any matrix of a plan: its Newton-Schulz runs on tiles of 128 x */
-#define THORN_MAT_TILES_256 128    /* 128 or 256 x 256 (a test hook: a plan chooses by itself) */
+#define THORN_MAT_TILES_256 128    /* 128 or 256 x 256 (a test hook: a plan chooses by itself); 128 not beside a
+                                      large matrix (short side > 256 or 2^20 elements) with MD or MD_SCALAR */
 
 /* Per-step flags (ThornOrthoMatStep.step_flags). */
 #define THORN_STEP_KEEP_GRAD 8     /* none_grad=False. No effect since ABI 5: the gradient of a

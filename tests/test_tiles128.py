@@ -24,6 +24,10 @@ def test_which_tiles_a_plan_takes():
     assert _tile([(300, 520)], _lib.MAT_MD) == 256     # its sums of p^2 follow the tiles
     assert _tile([(300, 520)], _lib.MAT_TILES_256) == 256
     assert _tile([(4096, 4096)], _lib.MAT_TILES_128) == 128
+    for md in (_lib.MAT_MD, _lib.MAT_MD_SCALAR):       # ... which the other kernel does not make
+        with pytest.raises(RuntimeError, match='TILES_128'):
+            _tile([(300, 520)], md | _lib.MAT_TILES_128)
+        assert _tile([(64, 96)], md | _lib.MAT_TILES_128) == 128
     # a matrix of the small path has no such tiles and does not count
     assert _tile(layer(768) * 20 + [(64, 96)] * 500) == 256
 

@@ -1,14 +1,14 @@
 // Newton-Schulz phase launches on 128 x 128 tiles (gfx950): the operations of ns_phase_kernel for
 // launches whose 256 x 256 tiles would leave most of the chip idle or spend it on padding.
 //
-// A 256 x 256 tile holds a CU for K / 32 * ~0.45 us plus ~9 us of prologue and epilogue. A group of
+// A 256 x 256 tile holds a CU for K / 32 * ~0.45 us plus about 14 us of launch, prologue and epilogue. A group of
 // mid-size matrices has fewer of them than CUs (48 matrices of 384 x 1536: 144 in a symmetric
 // product, of which 384 -> 512 padding is 44%), so its 18 dependent launches wait for one tile's
 // latency each. Here a block of 256 threads computes 128 x 128, two blocks to a CU: four times the
 // tiles, a quarter of the work and of the staging in each, no padding at multiples of 128. The price
 // is LDS traffic: each wave's 64 x 64 reads 1 KB of fragments per MFMA, the whole 128 B per clock
 // of a CU at the full MFMA rate, so on launches that fill the chip anyway the 256 x 256 engine is
-// faster (plan_tiles in thorn_abi.hip chooses per kind of operation).
+// faster (plan_tiles in thorn_abi.hip chooses one side for all launches of a plan).
 //
 // The data layout is ns_phase_kernel's: s x s matrices as packed upper triangles of 256 x 256 blocks
 // (SqPanel) with whole symmetric diagonal blocks. Of a diagonal block's four tiles the upper three
@@ -295,10 +295,10 @@ __device__ __forceinline__ void t128_sym(const OrthoMat& M, const NsOp& op, floa
 }
 
 // Epilogue of an update tile (see update_finish): the next iterate, u' and its row sums, or p.
-// tj: the tile's column, rows of rowsqpart; local: its number, of psqpart.
+// tj: the tile's column, rows of rowsqpart. (No sums of p^2: plans with decouple_md keep 256 x 256 tiles.)
 template <class T>
 __device__ __forceinline__ void t128_update(const OrthoMat& M, const NsOp& op, floatx16 (&acc)[T::N], int m0, int n0,
-                                            int tj, int local, char* smem) {
+                                            int tj, char* smem) {
     const int rows = M.rows, cols = M.cols, ldx = M.ldx, flags = M.flags;
     const float osc = op.first ? M.scal[kScalX0Scale] : 1.f;
     _Float16* const xout = op.xsel == kXA ? M.xb : M.xa;
@@ -355,12 +355,9 @@ __device__ __forceinline__ void t128_update(const OrthoMat& M, const NsOp& op, f
     }
     const bool apply = (flags & kFlagApply) != 0;
     const float eta = (flags & kFlagMagma) ? M.eta * ldg<float>(M.magma_s) : M.eta, wd = M.wd;
-    float psq = 0.f;
     auto step1 = [&](float x, float u) {
         const float q = cautious_step(x, u, eta, wd);
-        x = apply ? q : x;
-        psq += x * x;
-        return x;
+        return apply ? q : x;
     };
     auto step8 = [&](float (&v)[8], const half8v& h) {
 #pragma unroll
@@ -380,10 +377,6 @@ __device__ __forceinline__ void t128_update(const OrthoMat& M, const NsOp& op, f
         auto at = [&](int r, int c) { return reinterpret_cast<const _Float16*>(smem + t128_off(r, c)); };
         if (bf) update_edge<true, kT128>(rows_of, at, p, m0, n0, rows, cols, vec, apply, step1, step8);
         else update_edge<false, kT128>(rows_of, at, p, m0, n0, rows, cols, vec, apply, step1, step8);
-    }
-    if (flags & (kFlagMD | kFlagMDScalar)) {
-        const float t = block_sum(psq, reinterpret_cast<float*>(smem + T::TILE));
-        if (threadIdx.x == 0) M.psqpart[local] = t;
     }
 }
 
@@ -444,7 +437,7 @@ __global__ __launch_bounds__(T::NT, 2) void ns_phase128_kernel(const OrthoMat* _
     const bool on = update || ti != tj || T::a0(wave) < T::b0(wave) + 32 * T::NB;
     floatx16 acc[T::N];
     t128_gemm<T>(A, B, m0, n0, KT, a_k0, b_k0, ct, on, acc, smem);
-    if (update) t128_update<T>(M, op, acc, m0, n0, tj, local, smem);
+    if (update) t128_update<T>(M, op, acc, m0, n0, tj, smem);
     else t128_sym<T>(M, op, acc, on, m0, n0, smem);
 }
 

@@ -229,7 +229,7 @@ bool takes_small_path(int64_t rows, int64_t cols) {
 // width 1024 1595 and 1810, one 4096 x 4096 1496 and 2078, the Qwen3-300M set 6752 and 7916: the two
 // meet where 256 x 256 tiles give about half of the CUs one. Results are bit for bit the same, but for
 // decouple_md, whose sums of p^2 follow the tiles: such plans keep 256, so that a matrix's result does
-// not depend on the plan it is in.
+// not depend on the plan it is in (0: 128 was asked for all the same; ns_phase128_kernel makes no such sums).
 int plan_tiles(const ThornOrthoMatDesc* d, int n) {
     int forced = 0;
     bool md = false, square = true;
@@ -249,7 +249,7 @@ int plan_tiles(const ThornOrthoMatDesc* d, int n) {
         sym_k = std::max(sym_k, double(s));
         gram_k = std::max(gram_k, double(l));
     }
-    if (forced) return forced;
+    if (forced) return forced == 128 && md ? 0 : forced;
     if (md) return 256;
     auto time = [](int q, double N, double K) {
         if (!q) return std::max(1.0, N / 256) * (0.45 * K / 32 + 14);
@@ -666,6 +666,10 @@ int thorn_ortho_plan_create(const ThornOrthoMatDesc* descs, int n, thorn_ortho_p
         return o;
     };
     plan->tile = plan_tiles(descs, n);
+    if (plan->tile == 0) {
+        delete plan;
+        return fail(THORN_ERR_INVALID, "thorn_ortho_plan_create: TILES_128 excludes large matrices with MD or MD_SCALAR");
+    }
     const int tile = plan->tile;
     for (int i = 0; i < n; ++i) {
         const ThornOrthoMatDesc& d = descs[i];
