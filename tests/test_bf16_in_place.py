@@ -74,11 +74,17 @@ RESUMED = {'large': [(1024, 3072), (3072, 1024), (1000, 3072), (1024, 3070), (64
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize('group', RESUMED)
-def test_first_iterate_takes_the_unrounded_moment(group, monkeypatch):
-    print(f'[gpu] bf16 in place, resumed, {group}', flush=True)
+@pytest.mark.parametrize('group,tiles', [('large', 128), ('large', 256), ('small', 0)])
+def test_first_iterate_takes_the_unrounded_moment(group, tiles, monkeypatch):
+    print(f'[gpu] bf16 in place, resumed, {group}, tiles of {tiles}', flush=True)
     gen = torch.Generator().manual_seed(13)
     shapes = RESUMED[group]
+    shapes_of = OPT._plan_shapes
+
+    def forced(*args, **kw):   # (both sizes of tiles have a kernel of their own for the last update)
+        rows, cols, flags, *rest = shapes_of(*args, **kw)
+        flag = {128: _lib.MAT_TILES_128, 256: _lib.MAT_TILES_256, 0: 0}[tiles]
+        return (rows, cols, [f | flag for f in flags], *rest)
     start, moments = ([(torch.randn(s, generator=gen) * f).to(torch.bfloat16) for s in shapes] for f in (0.02, 2e-3))
     steps = [[(torch.randn(s, generator=gen) * f).to(torch.bfloat16) for s in shapes] for f in (1e-3, 1e-3, 0.1)]
 
@@ -87,6 +93,7 @@ def test_first_iterate_takes_the_unrounded_moment(group, monkeypatch):
             monkeypatch.setattr(OPT, '_needs_shadow', lambda p, group, state: p.dtype == torch.bfloat16)
         else:
             monkeypatch.undo()
+        monkeypatch.setattr(OPT, '_plan_shapes', forced)
         ps = [torch.nn.Parameter(t.to(DEV)) for t in start]
         opt = THORN([{'orthogonalize': True, 'params': ps, 'lr': 2e-2, 'betas': (0.9, 0.95)}])
         for p, m in zip(ps, moments):
@@ -104,6 +111,44 @@ def test_first_iterate_takes_the_unrounded_moment(group, monkeypatch):
     for k, (a, b) in enumerate(zip(run(False), run(True))):
         for s, x, y in zip(shapes * 2, a, b):
             assert torch.equal(x, y), (k, s, (x != y).sum().item())
+
+
+@pytest.mark.gpu
+def test_chains_in_place():
+    """A bf16 group that steps as two chains, each with its prologue on a stream of its own, against the same group
+    as one plan and as chains of working copies: a resumed run whose gradients jump in the third step (the first
+    iterate is made again from the moment before the step)."""
+    print('[gpu] bf16 in place, two chains', flush=True)
+    gen = torch.Generator().manual_seed(14)
+    shapes = [(384, 640), (640, 384), (512, 512), (1024, 384), (96, 640)] * 5 + [(3, 384, 512)]
+    start, moments = ([(torch.randn(s, generator=gen) * f).to(torch.bfloat16) for s in shapes] for f in (0.02, 2e-3))
+    steps = [[(torch.randn(s, generator=gen) * f).to(torch.bfloat16) for s in shapes] for f in (1e-3, 1e-3, 0.1)]
+
+    def run(chains, copies):
+        with pytest.MonkeyPatch.context() as mp:
+            mp.setattr(OPT, 'CHAIN_MIN_MATRICES', 16 if chains else 1 << 30)
+            mp.setattr(OPT, 'CHAIN_MIN_COST', 0)
+            if copies:
+                mp.setattr(OPT, '_needs_shadow', lambda p, group, state: True)
+            ps = [torch.nn.Parameter(t.to(DEV)) for t in start]
+            opt = THORN([{'orthogonalize': True, 'params': ps, 'lr': 2e-2, 'betas': (0.9, 0.95)}])
+            for p, m in zip(ps, moments):
+                opt.state[p].update(step=10, moment=m.to(DEV))
+            out = []
+            for grads in steps:
+                for p, g in zip(ps, grads):
+                    p.grad = g.to(DEV)
+                opt.step()
+                out.append([p.detach().clone() for p in ps] + [opt.state[p]['moment'].clone() for p in ps])
+            assert next(iter(opt._runners.values())).chained == chains and bool(opt._shadows) == copies
+            opt.check_status()
+            return out
+
+    chained = run(True, False)
+    for other in (run(False, False), run(True, True)):
+        for k, (a, b) in enumerate(zip(chained, other)):
+            for s, x, y in zip(shapes * 2, a, b):
+                assert torch.equal(x, y), (k, s, (x != y).sum().item())
 
 
 @pytest.mark.gpu

@@ -1,6 +1,6 @@
 """Matrices with a short side of at most 128, whose Newton-Schulz schedule runs in a workgroup's LDS
-(thin_schedule): one fused launch against the separate launches bit for bit, and both against the step in
-64 bits."""
+(thin_schedule): one fused launch against the separate launches bit for bit, both against the step in 64 bits,
+and thin matrices against larger ones that hold them."""
 import pytest
 import torch
 
@@ -37,7 +37,7 @@ def _exact(p, g, lr, wd):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16], ids=['fp32', 'bf16'])
-def test_fused_equals_separate_and_64_bits(dtype, monkeypatch):
+def test_fused_equals_separate_and_first_step_in_64_bits(dtype, monkeypatch):
     print(f'[gpu] thin matrices, {dtype}', flush=True)
     gen = torch.Generator().manual_seed(17)
     start = [(torch.randn(s, generator=gen) * 0.05).to(dtype) for s in SHAPES]
@@ -86,16 +86,8 @@ INSIDE = [((16, 3072), (129, 3072)), ((1, 300), (130, 300)), ((16, 4100), (140, 
           ((3999, 40), (3999, 160)), ((700, 47), (700, 188)), ((900, 33), (900, 132))]
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize('odd', [False, True], ids=['aligned', 'odd addresses'])
-def test_thin_sums_are_those_of_the_other_schedule(odd):
-    """Rows or columns of zeros change no sum, so a thin matrix steps bit for bit as the part of a larger one
-    that holds it: norms, Gram matrices (one chain over K, in one workgroup or dealt over a cluster), products
-    and the sums of per-row normalization (with four times the columns, exactly four times as large a divisor).
-    Odd addresses: the elementwise loads, where a width of no whole groups of four would take them in one of the
-    two alone."""
-    print(f'[gpu] thin matrices inside larger ones, odd addresses {odd}', flush=True)
-    pairs = [q for q in INSIDE if odd or q[0][1] % 4 == q[1][1] % 4]
+def _equals_inside(pairs, odd=False, **group):
+    """Steps of the matrices `pairs[i][0]` and of larger ones that hold them beside zeros, bit for bit the same."""
     gen = torch.Generator().manual_seed(23)
 
     def place(t, shape):
@@ -110,7 +102,7 @@ def test_thin_sums_are_those_of_the_other_schedule(odd):
 
     def run(shapes):
         ps = [torch.nn.Parameter(place(t, s)) for t, s in zip(start, shapes)]
-        opt = THORN([{'orthogonalize': True, 'params': ps, 'lr': 1e-2, 'weight_decay': 0.1}])
+        opt = THORN([{'orthogonalize': True, 'params': ps, 'lr': 1e-2, 'weight_decay': 0.1, **group}])
         for p, m, s in zip(ps, moments, shapes):
             opt.state[p].update(step=10, moment=place(m, s))
         out = []
@@ -124,7 +116,71 @@ def test_thin_sums_are_those_of_the_other_schedule(odd):
 
     for k, (a, b) in enumerate(zip(run([q for q, _ in pairs]), run([q for _, q in pairs]))):
         for (s, _), x, y in zip(pairs, a, b):
+            assert torch.isfinite(x).all(), (k, s)
             assert torch.equal(x, y), (k, s, (x != y).float().mean().item())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('odd', [False, True], ids=['aligned', 'odd addresses'])
+def test_thin_sums_are_those_of_the_other_schedule(odd):
+    """Rows or columns of zeros change no sum, so a thin matrix steps bit for bit as the part of a larger one
+    that holds it: norms, Gram matrices (one chain over K, in one workgroup or dealt over a cluster), products
+    and the sums of per-row normalization (with four times the columns, exactly four times as large a divisor).
+    Odd addresses: the elementwise loads, where a width of no whole groups of four would take them in one of the
+    two alone."""
+    print(f'[gpu] thin matrices inside larger ones, odd addresses {odd}', flush=True)
+    _equals_inside([q for q in INSIDE if odd or q[0][1] % 4 == q[1][1] % 4], odd)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('group', [dict(iters=2), dict(iters=3, lower_bound=1e-2), dict(iters=8, lower_bound=1e-1),
+                                   dict(iters=10, lower_bound=1e-6), dict(force_per_neuron_norm=True)], ids=str)
+def test_thin_matrices_under_other_options(group):
+    """Schedules of other lengths with one to three restarts, and per-row normalization of wide matrices."""
+    print(f'[gpu] thin matrices inside larger ones, {group}', flush=True)
+    _equals_inside([q for q in INSIDE if q[0][1] % 4 == q[1][1] % 4], **group)
+
+
+# small matrices with more rows than the fused launch keeps scales of in LDS (12288)
+TALL = [(12300, 40), (13000, 80), (20000, 50), (40000, 26)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('group', ['thin', 'tall'])
+def test_the_fused_launch_runs_and_gives_the_second_step(group):
+    """From its second step on, a plan of small matrices is one launch, and the second step's result is the
+    separate launches' and (to the iteration's bars) the 64-bit one."""
+    print(f'[gpu] the fused launch, {group}', flush=True)
+    shapes = [s for s in SHAPES if len(s) == 2] if group == 'thin' else TALL
+    gen = torch.Generator().manual_seed(29)
+    start = [torch.randn(s, generator=gen) * 0.05 for s in shapes]
+    steps = [[torch.randn(s, generator=gen) * 1e-3 for s in shapes] for _ in range(2)]
+    lr, wd = 1e-2, 0.1
+    ends = []
+    for fused in (True, False):
+        ps = [torch.nn.Parameter(t.to(DEV)) for t in start]
+        opt = THORN([{'orthogonalize': True, 'params': ps, 'lr': lr, 'weight_decay': wd}])
+        for k, grads in enumerate(steps):
+            before = [(p.detach().clone(), opt.state[p]['moment'].clone()) for p in ps] if k else None
+            for p, g in zip(ps, grads):
+                p.grad = g.to(DEV)
+            if k:
+                plan, = next(iter(opt._runners.values())).plans
+                plan.set_small_fusion(fused)
+                plan.timing_enable(64)
+            opt.step()
+        kinds = {name for name, (_, n) in plan.timing_read().items() if n}
+        assert kinds == {'small'} if fused else kinds > {'small', 'pre', 'norm', 'pnn_apply'}, kinds
+        opt.check_status()
+        ends.append([p.detach().clone() for p in ps])
+    for s, x, y in zip(shapes, *ends):
+        assert torch.equal(x, y), s
+    for s, (p, m), g, got in zip(shapes, before, steps[1], ends[0]):
+        g = g.to(DEV).double()
+        want = _exact(p, (g + 0.9 * (0.9 * m.double() + g)) / 1.9, lr, wd)
+        near = s[0] != s[1] and max(s) - min(s) <= 2
+        err = ((got.double() - want).norm() / (want - p.double()).norm()).item()
+        assert err <= (5e-2 if near else 2e-2), (s, err)
 
 
 @pytest.mark.gpu
