@@ -887,17 +887,17 @@ __device__ __forceinline__ void small_fused_apply(const OrthoMat& M, int member,
     float x[kKeepRounds][16];
 #pragma unroll
     for (int r = 0; r < kKeepRounds; ++r)
-        if (t0 + r * per < ntiles) pnn_load_p<BF>(M, t0 + r * per, t256, x[r]);
+        if (t0 + r * per < ntiles) tile_load<BF>(M, TileMap(M, t0 + r * per, t256), M.p, x[r]);
     float* const rows = reinterpret_cast<float*>(stages + kThinLds) - kSmallThreads;   // past sc
     const float gamma = pnn ? pnn_gamma(M, red, rows, staged ? sc : M.rowscale) : 1.f;   // its block_sum syncs them
     if (pnn && member == 0 && threadIdx.x == 0) M.scal[kScalGamma] = gamma;
     auto scale = [&](int row) { return staged ? sc[row] : ldg<float>(M.rowscale + row); };
 #pragma unroll
     for (int r = 0; r < kKeepRounds; ++r)
-        if (t0 + r * per < ntiles) (void)pnn_apply_p<BF>(M, t0 + r * per, t256, M.xa, gamma, scale, x[r]);
+        if (t0 + r * per < ntiles) pnn_apply_p<BF>(M, t0 + r * per, t256, M.xa, gamma, scale, x[r]);
     for (int t = t0 + kKeepRounds * per; t < ntiles; t += per) {
-        pnn_load_p<BF>(M, t, t256, x[0]);
-        (void)pnn_apply_p<BF>(M, t, t256, M.xa, gamma, scale, x[0]);
+        tile_load<BF>(M, TileMap(M, t, t256), M.p, x[0]);
+        pnn_apply_p<BF>(M, t, t256, M.xa, gamma, scale, x[0]);
     }
 }
 
