@@ -797,9 +797,9 @@ CHAIN_MAX_COST = 1e12
 # last less than the host takes to enqueue them twice. Measured as two chains and as one plan, each on
 # its better tiles: 40 matrices of width 320 506 and 414 us (2.5e9), 48 of 384 (and 12 squares) 936 and
 # 577 (8e9), 100 of 512 1272 and 1325 (2.2e10), 40 of 768 964 and 952 (3e10), 100 of 640 1407 and 1523
-# (4.3e10), 40 of 1024 1567 and 1595 (7e10), 100 of 768 1877 and 2080 (7.3e10). (Smaller groups keep
-# their two chains, which the tests of the chained step cover, though one plan is faster there as
-# well: 23 matrices of 384 to 1024 490 and 289 us.)
+# (4.3e10), 40 of 1024 1567 and 1595 (7e10), 100 of 768 1877 and 2080 (7.3e10). CHAIN_FEW_MATRICES is where
+# these measurements begin, not where the line ought to lie: groups of 16 to 31 keep the two chains they
+# had, and the one that was measured is faster as one plan as well (23 matrices of 384 to 1024, 490 and 289 us).
 CHAIN_FEW_MATRICES = 32
 CHAIN_MIN_COST = 2e10
 # Streams of the gradient-release steps (_release_step): with the caller's own, as many as the
